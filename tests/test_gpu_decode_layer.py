@@ -505,3 +505,36 @@ def test_two_decoder_layers_chained():
             h_dev_in = out
     finally:
         store.close()
+
+
+@pytest.mark.parametrize("ctx", [0, 1, 30, 31, 32, 62, 63, 64, 4096])
+@pytest.mark.parametrize("stale", [np.nan, np.inf])
+def test_decode_layer_slot_never_written(ctx, stale):
+    """The slot of the new token may hold anything before the call: the layer's
+    output and the pool are those of a zeroed slot, bit for bit."""
+    L = Layer(SMALL["n_embd"], SMALL["n_head"], SMALL["n_kv"], SMALL["hd"], SMALL["n_ff"], Q4KM, 4700)
+    kv_dim, n_blocks = L.n_kv * L.hd, ctx // BLOCK + 1
+    cfg = ssdq.layer_config(L.n_embd, L.n_head, L.n_kv, L.hd, L.n_ff, 10000.0, EPS)
+    nbytes, offs = ssdq.decode_layer_scratch(cfg)
+    hidden = synth.rng(4701).standard_normal(L.n_embd).astype(np.float32)
+    store = ssdq.WeightStore()
+    try:
+        L.upload(store, 0)
+        runs = []
+        for dirty in (False, True):
+            pool = Pool(kv_dim, ctx, n_blocks, n_blocks + 3, (1.0, 1.0), 4702)
+            if dirty:
+                r = pool.slot(ctx)
+                pool.kc[r * kv_dim:(r + 1) * kv_dim] = pool.vc[r * kv_dim:(r + 1) * kv_dim] = -128
+                pool.ks[r] = pool.vs[r] = stale
+            pool.upload()
+            announce("decode layer, slot never written", ctx, stale, dirty)
+            scratch = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+            out, got = run_gpu_layer(store, 0, cfg, hidden, ctx, pool, scratch, offs, step_sizes(L))
+            runs.append([out, got["attn"]] + pool.from_device())
+        assert np.all(np.isfinite(runs[0][0]))
+        for clean, dirty in zip(*runs):
+            assert bits_equal(clean, dirty)
+    finally:
+        store.close()
+        torch.cuda.synchronize()
