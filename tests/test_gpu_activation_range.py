@@ -2,14 +2,15 @@
 
 Real decoder hidden states carry a few channels 10^3-10^4 times larger than
 the rest, in many 32-element groups.  The matvec kernels carry x per
-32-element group as an integer of at most 2^30 against the group's largest
-magnitude, so an element 2^k below its group's maximum keeps 30 - k bits
+32-element group as an integer of at most 2^30 (batches: 2^30 or 2^31) against
+the group's largest magnitude, so an element 2^k below its group's maximum
+keeps 30 - k bits
 (with 22 bits, 3-9 of these 14336 outputs per case fell outside the
 tolerance).
 These cases check that the outputs still meet the stated tolerance against
 the reference's serial fp32 chain (matvec_*_cpu, src/metal/compute.rs:680-925),
 with the exact-sum substitution only where that chain is itself off, at the
-Llama-3-8B FFN shape 14336 x 4096 for Q4_K, Q4_0 and Q8_0, batch 1 and 8.
+Llama-3-8B FFN shape 14336 x 4096 for Q4_K, Q4_0, Q8_0 and Q6_K, batch 1 and 8.
 """
 import numpy as np
 import pytest
@@ -35,7 +36,7 @@ def massive_activations(batch, in_dim, seed, frac=0.01, lo=1e3, hi=1e4):
     return x, ch
 
 
-@pytest.mark.parametrize("dtype", [ssdq.Q4_K, ssdq.Q4_0, ssdq.Q8_0])
+@pytest.mark.parametrize("dtype", [ssdq.Q4_K, ssdq.Q4_0, ssdq.Q8_0, ssdq.Q6_K])
 @pytest.mark.parametrize("batch", [1, 8])
 def test_massive_activation_channels(dtype, batch):
     out_dim, in_dim = 14336, 4096

@@ -1,12 +1,15 @@
 """Batched matvec on the matrix cores (2-32 activation rows per pass).
 
-Bound: x is rounded once, by at most 2^-31 of its 256-element unit's largest
+Bound: x is rounded once, by at most 2^-31 of its 32-element block's largest
 magnitude rounded up to a power of two (at most twice that magnitude); all sums
 are integers or double, and the result is rounded once to fp32:
-|y - exact| <= 2^-24 |exact| + 2^-30 sum_units max|x_u| sum|w_u|.  The exact sum
+|y - exact| <= 2^-24 |exact| + 2^-30 sum_blocks max|x_b| sum|w_b|.  The exact sum
 here is of the reference's element values, which are rounded to fp32 (2^-24 of
 each); the kernel's are not: 2^-24 sum |w x| more, which also covers the double
-sums' own rounding.
+sums' own rounding.  Q6_K rows of an odd block count take the byte-addressed
+kernel, whose sums are fp32: chains of 16 elements, of at most K / 1024 + 1 such
+groups a lane and of 6 steps across the lanes, each step rounding by at most
+2^-24 sum |w x|.
 """
 import numpy as np
 import pytest
@@ -42,8 +45,10 @@ def close_to_exact(y, dtype, w, x, out_dim, in_dim):
     k = e.shape[1]
     x = x.astype(np.float64)[:, :k]
     exact = x @ e.T
-    mx = np.repeat(np.abs(x).reshape(len(x), k // 256, 256).max(axis=2), 256, axis=1)
+    mx = np.repeat(np.abs(x).reshape(len(x), k // 32, 32).max(axis=2), 32, axis=1)
     bound = 2.0 ** -24 * np.abs(exact) + 2.0 ** -30 * (mx @ np.abs(e).T) + 2.0 ** -24 * (np.abs(x) @ np.abs(e).T)
+    if dtype == Q6_K and k // 256 % 2:
+        bound += 2.0 ** -24 * (16 + k // 1024 + 1 + 6) * (np.abs(x) @ np.abs(e).T)
     err = np.abs(y.astype(np.float64).reshape(exact.shape) - exact)
     assert np.all(err <= bound), f"worst error / bound {np.nanmax(err / np.maximum(bound, 1e-300))}"
 
@@ -75,6 +80,39 @@ def test_batch_extreme_scales(dtype, lo, hi):
     announce("batch extreme scales", dtype)
     y = empty_dev(out_dim * batch, torch.float32)
     assert ssdq.matvec(dtype, to_dev(w), to_dev(x), y, out_dim, in_dim, batch) == 0
+    close_to_exact(from_dev(y), dtype, w, x, out_dim, in_dim)
+
+
+def without_weight(dtype, w):
+    """w with a zero weight for the first element of every 256 (and, Q4_K, no minima)."""
+    b = w.reshape(-1, synth.BLOCK[dtype][1]).copy()
+    if dtype == Q4_0:
+        b[::8, 2] = (b[::8, 2] & 0xF0) | 8
+    elif dtype == Q8_0:
+        b[::8, 2] = 0
+    elif dtype == Q4_K:
+        b[:, 2:4] = 0
+        b[:, 16] &= 0xF0
+    else:
+        b[:, 0] &= 0xF0
+        b[:, 128] = (b[:, 128] & 0xFC) | 2
+    return b.ravel()
+
+
+@pytest.mark.parametrize("dtype", [Q4_0, Q8_0, Q4_K, Q6_K])
+@pytest.mark.parametrize("batch", [2, 8, 13, 32])
+@pytest.mark.parametrize("large", [3e7, 1e20])
+def test_batch_large_channel_without_weight(dtype, batch, large):
+    # a channel far above the rest of its 256 elements, and of no weight: the blocks it is not in keep their precision
+    out_dim, in_dim = 100, 1024
+    w = without_weight(dtype, synth.quant_weights(dtype, out_dim, in_dim, 7400))
+    x = synth.normal_f32((batch, in_dim), 7401).reshape(batch, in_dim).copy()
+    x[:, ::256] = large
+    x[:, 1:32] = x[:, 257:288] = x[:, 513:544] = x[:, 769:800] = 0  # its own block
+    announce("batch large channel", dtype, batch, large)
+    y = empty_dev(out_dim * batch, torch.float32)
+    assert ssdq.matvec(dtype, to_dev(w), to_dev(x), y, out_dim, in_dim, batch) == 0
+    x[:, ::256] = 0
     close_to_exact(from_dev(y), dtype, w, x, out_dim, in_dim)
 
 
