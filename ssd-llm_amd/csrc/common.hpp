@@ -204,6 +204,31 @@ __device__ __forceinline__ void planes4(uint32_t a, uint32_t b, uint32_t c, uint
   out[3] = __builtin_amdgcn_perm(ce_hi, ab_hi, 0x07060302u);
 }
 
+// 4 x 4 transpose of one dword of four sources held by the four 16-lane rows:
+// on entry lane row r holds v[i] = dword i of source r; on exit v[i] = dword r
+// of source i.
+__device__ __forceinline__ void transpose4(uint32_t (&v)[4]) {
+  const auto p01 = __builtin_amdgcn_permlane16_swap(v[0], v[1], false, false);
+  const auto p23 = __builtin_amdgcn_permlane16_swap(v[2], v[3], false, false);
+  const auto q02 = __builtin_amdgcn_permlane32_swap(p01[0], p23[0], false, false);
+  const auto q13 = __builtin_amdgcn_permlane32_swap(p01[1], p23[1], false, false);
+  v[0] = q02[0];
+  v[1] = q13[0];
+  v[2] = q02[1];
+  v[3] = q13[1];
+}
+
+// A dword of each lane row (v of lane row r in out[r]) to every row.
+__device__ __forceinline__ void from_rows(uint32_t v, uint32_t (&out)[4]) {
+  const auto t = __builtin_amdgcn_permlane16_swap(v, v, false, false);  // rows 0 0 2 2, 1 1 3 3
+  const auto t0 = __builtin_amdgcn_permlane32_swap(t[0], t[0], false, false);
+  const auto t1 = __builtin_amdgcn_permlane32_swap(t[1], t[1], false, false);
+  out[0] = t0[0];
+  out[1] = t1[0];
+  out[2] = t0[1];
+  out[3] = t1[1];
+}
+
 // INT8 code of one KV element (quantize_vectors_int8, src/ssd/block_swap.rs:36-60
 // = QuantizedVec::quantize, src/inference/quantized_kv_cache.rs:23-41):
 // clamp(round_half_away(v * inv), -127, 127), NaN -> 0 (Rust `as i8`), as a

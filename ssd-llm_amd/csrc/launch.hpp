@@ -184,6 +184,12 @@ hipError_t launch_flash_attn_f32(const float* q, const float* k, const float* v,
                                  int window_start, int window_end, void* workspace,
                                  hipStream_t stream);
 
+// Q8_0 matvec of 2-8 activation rows on the matrix cores (matvec_mfma.hip);
+// hipErrorNotSupported when the shape or alignment does not fit it.
+bool q8_mfma_supported(const void* w, const float* x, size_t in_dim, size_t batch);
+hipError_t launch_q8_mfma(const uint8_t* w, const float* x, float* y, size_t out_dim, size_t in_dim, size_t batch,
+                          hipStream_t s);
+
 // Matvec of 2 .. kBatchMfmaMax activation rows on the matrix cores (Q4_0, Q8_0,
 // Q4_K, Q6_K; matvec_batch.hip); hipErrorNotSupported when the operands do not
 // fit it or the workspace is smaller than its K slices need.

@@ -2582,9 +2582,10 @@ hipError_t fast_dispatch(const uint8_t* w, const float* x, float* y, int out_dim
     if (e != hipSuccess || *used) return e;
   } else {
     // chunks of up to 32 activation rows on the matrix cores (of up to 8 when
-    // the workspace holds no more); rows of Q4_0 / Q8_0 that are not whole
-    // 256-element units in chunks of 8 / 4 / 2 on mv_bn; a last single row on
-    // mv_b1 (the first chunk decides: every chunk has the same row geometry)
+    // the workspace holds no more); 2-8 rows of Q8_0 at K = 1024 / 2048 / 4096 on
+    // their own kernel there; rows of Q4_0 / Q8_0 that are not whole 256-element
+    // units in chunks of 8 / 4 / 2 on mv_bn; a last single row on mv_b1 (the
+    // first chunk decides: every chunk has the same row geometry)
     int b0 = 0;
     while (b0 < batch) {
       const int left = batch - b0;
@@ -2593,7 +2594,12 @@ hipError_t fast_dispatch(const uint8_t* w, const float* x, float* y, int out_dim
       bool u = false;
       hipError_t e = hipErrorNotSupported;
       int take = 1;
-      if (left >= 2 && batch_mfma_ok(F, w, xb, in_dim)) {
+      if (F == kQ8_0 && q8_mfma_supported(w, xb, in_dim, left)) {
+        take = left;
+        e = launch_q8_mfma(w, xb, yb, out_dim, in_dim, take, s);
+        u = e == hipSuccess;
+        if (e == hipErrorNotSupported) e = hipSuccess;
+      } else if (left >= 2 && batch_mfma_ok(F, w, xb, in_dim)) {
         for (int most : {(int)kBatchMfmaMax, 8}) {
           take = std::min(left, most);
           e = launch_batch_mfma(F, w, xb, yb, out_dim, in_dim, take, s, ws, ws_floats * sizeof(float));
@@ -2736,6 +2742,7 @@ size_t matvec_workspace_wanted(int dtype, const void* w, const float* x, size_t 
                                size_t in_dim, size_t batch) {
   const size_t n = matvec_workspace_bytes(dtype, w, x, out_dim, in_dim, batch);
   if (out_dim == 0 || batch < 2 || !batch_mfma_ok(dtype, w, x, in_dim)) return n;
+  if (dtype == kQ8_0 && q8_mfma_supported(w, x, in_dim, batch)) return n;
   return std::max(n, batch_mfma_workspace_bytes(out_dim, in_dim, std::min(batch, kBatchMfmaMax)));
 }
 
