@@ -2686,6 +2686,19 @@ size_t ws_floats_for(int od, int bpr, size_t batch) {
   return n;
 }
 
+// fast_aligned of the four types of launch_matvec.
+bool fast_aligned_type(int dtype, const void* w, const float* x, size_t in_dim) {
+  const uint8_t* wb = (const uint8_t*)w;
+  const int id = (int)in_dim;
+  switch (dtype) {
+    case kQ4_0: return fast_aligned<kQ4_0>(wb, x, id, id / 32);
+    case kQ8_0: return fast_aligned<kQ8_0>(wb, x, id, id / 32);
+    case kQ4_K: return fast_aligned<kQ4_K>(wb, x, id, id / 256);
+    case kQ6_K: return fast_aligned<kQ6_K>(wb, x, id, id / 256);
+    default: return false;
+  }
+}
+
 size_t matvec_digit_ext_workspace_bytes(int dtype, const void* w, const float* x, size_t out_dim, size_t in_dim,
                                         size_t batch) {
   if (out_dim == 0 || batch == 0) return 0;
@@ -2724,24 +2737,25 @@ hipError_t launch_matvec_digit_ext(int dtype, const uint8_t* w, const float* x, 
 
 size_t matvec_workspace_bytes(int dtype, const void* w, const float* x, size_t out_dim,
                               size_t in_dim, size_t batch) {
-  if (batch == 0 || out_dim == 0) return 0;
-  const uint8_t* wb = (const uint8_t*)w;
+  if (batch == 0 || out_dim == 0 || !fast_aligned_type(dtype, w, x, in_dim)) return 0;
   const int od = (int)out_dim, id = (int)in_dim;
   size_t n = 0;
   switch (dtype) {
-    case kQ4_0: if (fast_aligned<kQ4_0>(wb, x, id, id / 32)) n = ws_floats_for<kQ4_0>(od, id / 32, batch); break;
-    case kQ8_0: if (fast_aligned<kQ8_0>(wb, x, id, id / 32)) n = ws_floats_for<kQ8_0>(od, id / 32, batch); break;
-    case kQ4_K: if (fast_aligned<kQ4_K>(wb, x, id, id / 256)) n = ws_floats_for<kQ4_K>(od, id / 256, batch); break;
-    case kQ6_K: if (fast_aligned<kQ6_K>(wb, x, id, id / 256)) n = ws_floats_for<kQ6_K>(od, id / 256, batch); break;
+    case kQ4_0: n = ws_floats_for<kQ4_0>(od, id / 32, batch); break;
+    case kQ8_0: n = ws_floats_for<kQ8_0>(od, id / 32, batch); break;
+    case kQ4_K: n = ws_floats_for<kQ4_K>(od, id / 256, batch); break;
+    case kQ6_K: n = ws_floats_for<kQ6_K>(od, id / 256, batch); break;
     default: break;
   }
   return n * sizeof(float);
 }
 
+// Asks for the batched kernel's K slices only where fast_dispatch takes it.
 size_t matvec_workspace_wanted(int dtype, const void* w, const float* x, size_t out_dim,
                                size_t in_dim, size_t batch) {
   const size_t n = matvec_workspace_bytes(dtype, w, x, out_dim, in_dim, batch);
-  if (out_dim == 0 || batch < 2 || !batch_mfma_ok(dtype, w, x, in_dim)) return n;
+  if (out_dim == 0 || batch < 2 || !fast_aligned_type(dtype, w, x, in_dim) || !batch_mfma_ok(dtype, w, x, in_dim))
+    return n;
   if (dtype == kQ8_0 && q8_mfma_supported(w, x, in_dim, batch)) return n;
   return std::max(n, batch_mfma_workspace_bytes(out_dim, in_dim, std::min(batch, kBatchMfmaMax)));
 }

@@ -7,6 +7,8 @@ write live memory and still produce the oracle's result.  Tolerance: the
 matvec bar, |gpu - ref| <= 1e-4 + 1e-3 |ref| (with the exact-sum substitution
 of helpers.assert_close_attributed).
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -78,3 +80,28 @@ def test_graph_replay_after_workspace_growth():
     del g
     torch.cuda.synchronize()
     ssdq.release_workspaces()
+
+
+def test_no_workspace_for_calls_that_use_none():
+    # Q6_K rows of an odd block count run on the byte-addressed kernel, 2-8 rows of
+    # Q8_0 at K = 4096 in one launch: neither has K slices, so a stream of its own
+    # gets no workspace for them
+    hip = ctypes.CDLL("libamdhip64.so")
+    handle = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+    side = torch.cuda.ExternalStream(handle.value)
+    try:
+        for dtype, out_dim, in_dim, batch in ((ssdq.Q6_K, 4096, 11008, 32), (ssdq.Q8_0, 256, 4096, 8)):
+            w = to_dev(synth.quant_weights(dtype, out_dim, in_dim, 910))
+            x = to_dev(synth.normal_f32((batch, in_dim), 911))
+            y = torch.empty(batch * out_dim, dtype=torch.float32, device="cuda")
+            ssdq.matvec(dtype, w, x, y, 16, in_dim, 2)  # code loaded
+            torch.cuda.synchronize()
+            announce("workspace: none wanted", dtype, out_dim, in_dim, batch)
+            free = torch.cuda.mem_get_info()[0]
+            ssdq.matvec(dtype, w, x, y, out_dim, in_dim, batch, stream=side)
+            side.synchronize()
+            assert torch.cuda.mem_get_info()[0] == free
+    finally:
+        torch.cuda.synchronize()
+        hip.hipStreamDestroy(handle)
