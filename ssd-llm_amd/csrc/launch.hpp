@@ -194,12 +194,11 @@ hipError_t launch_q8_mfma(const uint8_t* w, const float* x, float* y, size_t out
 // Q4_K, Q6_K; matvec_batch.hip); hipErrorNotSupported when the operands do not
 // fit it or the workspace is smaller than its K slices need.
 constexpr size_t kBatchMfmaMax = 32;
+constexpr size_t kBatchWorkspaceMax = (size_t)32 << 20;
 bool batch_mfma_ok(int dtype, const void* w, const float* x, size_t in_dim);
 size_t batch_mfma_workspace_bytes(size_t out_dim, size_t in_dim, size_t nb);
 hipError_t launch_batch_mfma(int dtype, const uint8_t* w, const float* x, float* y, size_t out_dim, size_t in_dim,
                              size_t nb, hipStream_t s, void* workspace, size_t workspace_bytes);
-// y[i] = sum over slices z of part[z * n + i], in slice order (double partials).
-hipError_t launch_slice_reduce(const double* part, float* y, int n, int slices, hipStream_t s);
 
 // Prefill GEMM: Y_i[M,n_i] f32 = X[M,K] bf16 x W_i[n_i,K] Q4_K (reference
 // layout) for count = 1..3 matrices sharing X, computed as one GEMM.

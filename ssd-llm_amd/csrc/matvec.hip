@@ -2554,7 +2554,10 @@ hipError_t bn_dispatch(const uint8_t* w, const float* x, float* y, int out_dim, 
   if (e != hipSuccess) return e;
   *used = true;
   if (p.slices == 1) return hipSuccess;
-  return launch_slice_reduce(reinterpret_cast<const double*>(ws), y, NB * out_dim, p.slices, s);
+  const int n = NB * out_dim;
+  hipLaunchKernelGGL(slice_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+                     reinterpret_cast<const double*>(ws), y, n, p.slices, nullptr, nullptr);
+  return hipGetLastError();
 }
 
 // The batch-1 digit-plane kernel alone, for the types whose float path is
@@ -2758,12 +2761,6 @@ size_t matvec_workspace_wanted(int dtype, const void* w, const float* x, size_t 
     return n;
   if (dtype == kQ8_0 && q8_mfma_supported(w, x, in_dim, batch)) return n;
   return std::max(n, batch_mfma_workspace_bytes(out_dim, in_dim, std::min(batch, kBatchMfmaMax)));
-}
-
-hipError_t launch_slice_reduce(const double* part, float* y, int n, int slices, hipStream_t s) {
-  hipLaunchKernelGGL(slice_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, part, y, n, slices,
-                     nullptr, nullptr);
-  return hipGetLastError();
 }
 
 hipError_t launch_matvec_acc(int dtype, const uint8_t* w, const float* x, float* acc, float* y, size_t out_dim,

@@ -82,26 +82,54 @@ def test_graph_replay_after_workspace_growth():
     ssdq.release_workspaces()
 
 
+def own_stream():
+    """A stream that had no call before (torch hands out streams of a pool); kept,
+    so that no later stream gets its handle, and with it its workspace."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    handle = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+    return torch.cuda.ExternalStream(handle.value)
+
+
+def test_batch_workspace_is_bounded():
+    # 32 rows of a wide matrix with K slices: the partial sums of at most 32 MiB of
+    # rows at a time (43680 here), whole groups of 16, the last piece ragged
+    dtype, out_dim, in_dim, batch = ssdq.Q4_0, 90005, 2304, 32
+    w = synth.quant_weights(dtype, out_dim, in_dim, 920)
+    x = synth.normal_f32((batch, in_dim), 921).reshape(batch, in_dim)
+    wd, xd = to_dev(w), to_dev(x)
+    y = torch.empty(batch * out_dim, dtype=torch.float32, device="cuda")
+    ssdq.matvec(dtype, wd, xd, y, 16, in_dim, 2)  # code loaded
+    y.fill_(float("nan"))
+    torch.cuda.synchronize()
+    side = own_stream()
+    announce("workspace: bounded", out_dim, in_dim, batch)
+    free = torch.cuda.mem_get_info()[0]
+    ssdq.matvec(dtype, wd, xd, y, out_dim, in_dim, batch, stream=side)
+    side.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 34 << 20
+    y = y.cpu().numpy().reshape(batch, out_dim)
+    rows = np.r_[0:40, 43660:43700, 87340:87380, 89990:out_dim]
+    wr = w.reshape(out_dim, -1)[rows].ravel()
+    for b in (0, 31):
+        ref = o.matvec(dtype, wr, x[b], rows.size, in_dim)[0]
+        assert_close_attributed(y[b, rows], ref, o.matvec_exact(dtype, wr, x[b], rows.size, in_dim), f"row {b}")
+    assert np.isfinite(y).all()
+
+
 def test_no_workspace_for_calls_that_use_none():
     # Q6_K rows of an odd block count run on the byte-addressed kernel, 2-8 rows of
     # Q8_0 at K = 4096 in one launch: neither has K slices, so a stream of its own
     # gets no workspace for them
-    hip = ctypes.CDLL("libamdhip64.so")
-    handle = ctypes.c_void_p()
-    assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
-    side = torch.cuda.ExternalStream(handle.value)
-    try:
-        for dtype, out_dim, in_dim, batch in ((ssdq.Q6_K, 4096, 11008, 32), (ssdq.Q8_0, 256, 4096, 8)):
-            w = to_dev(synth.quant_weights(dtype, out_dim, in_dim, 910))
-            x = to_dev(synth.normal_f32((batch, in_dim), 911))
-            y = torch.empty(batch * out_dim, dtype=torch.float32, device="cuda")
-            ssdq.matvec(dtype, w, x, y, 16, in_dim, 2)  # code loaded
-            torch.cuda.synchronize()
-            announce("workspace: none wanted", dtype, out_dim, in_dim, batch)
-            free = torch.cuda.mem_get_info()[0]
-            ssdq.matvec(dtype, w, x, y, out_dim, in_dim, batch, stream=side)
-            side.synchronize()
-            assert torch.cuda.mem_get_info()[0] == free
-    finally:
+    side = own_stream()
+    for dtype, out_dim, in_dim, batch in ((ssdq.Q6_K, 4096, 11008, 32), (ssdq.Q8_0, 256, 4096, 8)):
+        w = to_dev(synth.quant_weights(dtype, out_dim, in_dim, 910))
+        x = to_dev(synth.normal_f32((batch, in_dim), 911))
+        y = torch.empty(batch * out_dim, dtype=torch.float32, device="cuda")
+        ssdq.matvec(dtype, w, x, y, 16, in_dim, 2)  # code loaded
         torch.cuda.synchronize()
-        hip.hipStreamDestroy(handle)
+        announce("workspace: none wanted", dtype, out_dim, in_dim, batch)
+        free = torch.cuda.mem_get_info()[0]
+        ssdq.matvec(dtype, w, x, y, out_dim, in_dim, batch, stream=side)
+        side.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free
