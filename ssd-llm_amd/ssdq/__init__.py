@@ -153,7 +153,15 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
-_raw_stream = None  # (initialised?, current device, its current stream's handle), from torch
+_raw_stream = None  # torch's _stream_calls
+
+
+def _stream_calls(torch):
+    """(initialised?, current device, its current stream's handle), as calls."""
+    try:
+        return torch.cuda.is_initialized, torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+    except AttributeError:  # private names: without them, the public call
+        return lambda: True, lambda: None, lambda _: torch.cuda.current_stream().cuda_stream
 
 
 def _stream(stream=None):
@@ -167,7 +175,7 @@ def _stream(stream=None):
         return stream.cuda_stream
     if _raw_stream is None:
         import torch
-        _raw_stream = (torch.cuda.is_initialized, torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+        _raw_stream = _stream_calls(torch)
     initialised, device, handle = _raw_stream
     if not initialised():
         import torch
