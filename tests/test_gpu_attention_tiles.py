@@ -35,7 +35,7 @@ def test_paged_tiles(n_head, n_kv, hd, ctx):
 
 
 def test_paged_value_scales_of_all_sizes():
-    # p * v_scale is rounded against the tile's largest: rows of very different scales in one tile
+    # rows of very different scales in one tile
     n_head, n_kv, hd, bs, ctx = 8, 2, 128, 16, [100]
     q, kc, ks, vc, vs, tables, cl = paged_case(1, n_head, n_kv, hd, bs, ctx, 7, 77)
     vs = np.asarray(vs) * np.float32(10.0) ** np.resize(np.arange(-6, 3), np.asarray(vs).shape).astype(np.float32)
@@ -44,6 +44,62 @@ def test_paged_value_scales_of_all_sizes():
     got, _ = run_paged(q, kc, ks, vc, vs, tables, cl, 1, n_head, n_kv, hd, bs, 7)
     ref = o.paged_attention_int8(q, kc, ks, vc, vs, tables, cl, 1, n_head, n_kv, hd, bs, 7)
     assert_close(got, ref, "paged value scales")
+
+
+def paged_softmax(q, kc, ks, tables, bs, ctx, n_kv):
+    """Weights of sequence 0's tokens [n_head, ctx] and their pool rows, in float64."""
+    hd = q.shape[2]
+    rows = tables.reshape(-1)[np.arange(ctx) // bs] * bs + np.arange(ctx) % bs
+    k = (kc.reshape(-1, n_kv, hd)[rows].astype(np.float64) * ks[rows].astype(np.float64)[:, None, None])
+    s = np.stack([k[:, h * n_kv // q.shape[1]] @ q[0, h].astype(np.float64) for h in range(q.shape[1])]) / np.sqrt(hd)
+    p = np.exp(s - s.max(axis=1, keepdims=True))
+    return p / p.sum(axis=1, keepdims=True), rows
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("ctx", [31, 64, 200])
+def test_paged_dimensions_of_low_weight_tokens(hd, ctx):
+    """Dimensions in which every token of more than 2^-35 of the largest weight has
+    value code 0 keep fp32's relative precision.  Bound, relative to sum p |v| of
+    the dimension: scores of magnitude up to 64 take four fp32 roundings (and so
+    does the largest, subtracted from them), which the exponential turns into
+    2 x 64 x 4 x 2^-24 = 3.1e-5; its own error, the sums' and the final division's
+    add less than 2e-6."""
+    n_head, n_kv, bs, mb = 4, 1, 16, 13
+    q, kc, ks, vc, vs, tables, cl = paged_case(1, n_head, n_kv, hd, bs, [ctx], mb, 90 + hd)
+    q[0, 1:] = q[0, :1] * np.array([0.9, 1.05, 1.1], np.float32)[:, None]  # one order of the tokens for all heads
+    p, rows = paged_softmax(q, kc, ks, tables, bs, ctx, n_kv)
+    q *= np.float32(40 / (np.log(p[0].max()) - np.log(np.median(p[0]))))
+    p, rows = paged_softmax(q, kc, ks, tables, bs, ctx, n_kv)
+    v = vc.reshape(-1, hd)
+    heavy = (p > 2.0 ** -35 * p.max(axis=1, keepdims=True)).any(axis=0)
+    assert 0 < heavy.sum() < ctx
+    dims = np.arange(0, hd, 3)
+    v[np.ix_(rows[heavy], dims)] = 0
+    announce("paged dimensions of low-weight tokens", hd, ctx)
+    got, _ = run_paged(q, kc, ks, v.reshape(-1), vs, tables, cl, 1, n_head, n_kv, hd, bs, mb)
+    vf = v[rows].astype(np.float64) * vs[rows].astype(np.float64)[:, None]
+    exact, size = p @ vf, p @ np.abs(vf)
+    assert size[:, dims].max() < 1e-6 and size[:, dims].min() > 0
+    err = np.abs(got.reshape(n_head, hd) - exact) / size
+    assert err.max() < 3.3e-5, err.max()
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("ctx,at", [(70, 3), (70, 69), (64, 63), (33, 32)])
+def test_paged_infinite_value_scale(hd, ctx, at):
+    # an infinite scale gives its token's codes their infinities, also where a ragged tile repeats the last token
+    n_head, n_kv, bs, mb = 4, 1, 16, 5
+    q, kc, ks, vc, vs, tables, cl = paged_case(1, n_head, n_kv, hd, bs, [ctx], mb, 95)
+    row = int(tables.reshape(-1)[at // bs]) * bs + at % bs
+    v = vc.reshape(-1, hd)
+    v[row] = np.where(np.arange(hd) % 2, 100, -7)
+    vs = vs.copy()
+    vs[row] = np.inf
+    announce("paged infinite value scale", hd, ctx, at)
+    got, _ = run_paged(q, kc, ks, v.reshape(-1), vs, tables, cl, 1, n_head, n_kv, hd, bs, mb)
+    want = np.where(np.arange(hd) % 2, np.inf, -np.inf)
+    assert (got.reshape(n_head, hd) == want).all()
 
 
 @pytest.mark.parametrize("n_head,n_kv,hd", [(4, 4, 128), (32, 8, 128), (10, 2, 128), (16, 1, 64), (3, 3, 256), (8, 2, 256)])
