@@ -196,7 +196,7 @@ hipError_t launch_q8_mfma(const uint8_t* w, const float* x, float* y, size_t out
 constexpr size_t kBatchMfmaMax = 32;
 constexpr size_t kBatchWorkspaceMax = (size_t)32 << 20;
 bool batch_mfma_ok(int dtype, const void* w, const float* x, size_t in_dim);
-size_t batch_mfma_workspace_bytes(size_t out_dim, size_t in_dim, size_t nb);
+size_t batch_mfma_workspace_bytes(int dtype, size_t out_dim, size_t in_dim, size_t nb);
 hipError_t launch_batch_mfma(int dtype, const uint8_t* w, const float* x, float* y, size_t out_dim, size_t in_dim,
                              size_t nb, hipStream_t s, void* workspace, size_t workspace_bytes);
 

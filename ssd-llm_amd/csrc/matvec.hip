@@ -2760,7 +2760,7 @@ size_t matvec_workspace_wanted(int dtype, const void* w, const float* x, size_t 
   if (out_dim == 0 || batch < 2 || !fast_aligned_type(dtype, w, x, in_dim) || !batch_mfma_ok(dtype, w, x, in_dim))
     return n;
   if (dtype == kQ8_0 && q8_mfma_supported(w, x, in_dim, batch)) return n;
-  return std::max(n, batch_mfma_workspace_bytes(out_dim, in_dim, std::min(batch, kBatchMfmaMax)));
+  return std::max(n, batch_mfma_workspace_bytes(dtype, out_dim, in_dim, std::min(batch, kBatchMfmaMax)));
 }
 
 hipError_t launch_matvec_acc(int dtype, const uint8_t* w, const float* x, float* acc, float* y, size_t out_dim,

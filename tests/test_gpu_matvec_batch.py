@@ -30,6 +30,8 @@ CASES = [  # (dtype, out_dim, in_dim, batch)
     (Q4_K, 300, 1024, 9), (Q6_K, 300, 1024, 16), (Q4_0, 300, 1024, 17), (Q8_0, 300, 1024, 32),
     # odd numbers of Q6_K blocks, which stay on the byte-addressed kernel
     (Q6_K, 7, 768, 3), (Q6_K, 1001, 1280, 6),
+    # few rows: one slice below 64 row units, more from there on (Q6_K: from 16 units on)
+    (Q4_K, 500, 4096, 3), (Q4_K, 500, 4096, 4), (Q6_K, 500, 3840 + 256, 2), (Q6_K, 500, 3584, 2), (Q4_0, 20, 2048, 16),
     # uneven units per wave and uneven K slices (9 and 33 units, 43 units at 8 / 32 rows)
     (Q4_K, 4097, 2304, 8), (Q4_0, 100, 8448, 4), (Q8_0, 100, 8448, 2), (Q4_K, 513, 11008, 7), (Q6_K, 129, 11008, 31),
     # more groups than waves (one wave walks several groups), chunks of 32 and a rest, a last single row
