@@ -457,10 +457,13 @@ __global__ __launch_bounds__((64 * kMaxWaves<F, B>)) void mv_ext(
     s += dpp_mov<0xB1>(s);  // lane i ^ 1, as shfl_xor(s, 1)
     if ((part & 1) == 0) xsum[((size_t)b * G + g) * 2 + (part >> 1)] = s;
   }
-  // orders LDS only: the first weights stay in flight
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  if constexpr (PF) {  // orders LDS only: the first weights stay in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  } else {
+    __syncthreads();
+  }
 
   for (int r0 = r_begin + wave * R; r0 < r_end; r0 += nwaves * R) {
     float acc[R][B];
@@ -510,9 +513,10 @@ __global__ __launch_bounds__((64 * kMaxWaves<F, B>)) void mv_ext(
       }
     } else {
       // The lanes walk in step, past the end too with groups that are not summed,
-      // since PF's loads belong to the next groups; BF16 without PF lets a lane
-      // stop at its last group (14336 x 4096: 22.0 us against 22.5).
-      constexpr bool kOwnEnd = !PF && F == kBF16;
+      // since PF's loads belong to the next groups; without PF, BF16 (14336 x 4096:
+      // 22.0 us against 22.5) and batches (IQ4_XS, two rows: 20.2 against 20.8) let
+      // a lane stop at its last group.
+      constexpr bool kOwnEnd = !PF && (F == kBF16 || B > 1);
       for (int g0 = kOwnEnd ? lane : 0; g0 < G; g0 += 64) {
         const int g = kOwnEnd ? g0 : min(g0 + lane, G - 1);
         const bool live = kOwnEnd || g0 + lane < G;
@@ -725,11 +729,15 @@ template <int F, int B, int R>
 hipError_t run_ext(const uint8_t* w, const float* x, float* y, int out_dim, int in_dim, int G,
                    size_t row_bytes, size_t lds, hipStream_t s) {
   if constexpr (!kPairGroups<F>) {
-    // PF's registers leave five workgroups of four waves to a CU: it is taken
-    // where no more fit for LDS (on rows of more than two groups a lane; at
-    // 14336 x 4096, two rows, it is 21.4 us against 20.3) or are there to run
+    // PF's registers leave five workgroups of four waves to a CU: at one row it is
+    // taken where no more fit for LDS (on rows of more than two groups a lane) or
+    // are there to run.  Two rows: BF16 alone, and of the few only up to one a CU
+    // (2048 x 4096 7.2 us against 8.0, 4096 x 4096 11.2 against 10.8; IQ4_XS 4096 x
+    // 8192 14.7 against 13.6, 512 x 4096 5.9 against 5.4); more rows: not taken
+    // (BF16 4096 x 4096, four rows 21.6 against 20.5)
     const int fit = ext_lds_limit() / (int)lds, need = (out_dim + 4 * R - 1) / (4 * R);
-    if ((fit <= 5 && G > 128) || need <= 5 * device_cu_count())
+    if ((B == 1 || (B == 2 && F == kBF16)) &&
+        ((fit <= 5 && G > 128) || need <= (B == 1 ? 5 : 1) * device_cu_count()))
       return run_ext_as<F, B, R, true>(w, x, y, out_dim, in_dim, G, row_bytes, lds, s);
   }
   return run_ext_as<F, B, R, false>(w, x, y, out_dim, in_dim, G, row_bytes, lds, s);
