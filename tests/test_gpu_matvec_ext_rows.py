@@ -37,6 +37,9 @@ def call(dtype, w, x, out_dim, in_dim, batch):
     (ssdq.IQ4_NL, 8195, 14336, 1),   # paired groups, 8 waves
     (ssdq.IQ3_S, 8195, 14336, 1),
     (ssdq.F16, 2051, 4096, 8),
+    (ssdq.BF16, 4601, 4096, 4),      # 5 waves, 9 rows a place
+    (ssdq.IQ3_S, 7001, 4096, 4),     # 7 waves
+    (ssdq.IQ4_XS, 9001, 14336, 1),   # 5 waves of two rows, 18 rows a place
     (ssdq.BF16, 1021, 4096, 2),      # two rows: requested ahead
     (ssdq.BF16, 4099, 4096, 2),      # too many rows for that
     (ssdq.IQ4_XS, 1021, 4352, 2),    # lanes stop at their own last group, 136 groups
