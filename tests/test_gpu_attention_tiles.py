@@ -102,6 +102,21 @@ def test_paged_infinite_value_scale(hd, ctx, at):
     assert (got.reshape(n_head, hd) == want).all()
 
 
+@pytest.mark.parametrize("ctx", [[3000, 100, 1, 0], [20000, 30, 6000]])
+def test_paged_records_of_an_earlier_call(ctx):
+    # short sequences have no records for the later splits: what an earlier call left there (infinities and NaN) is
+    # loaded with the rest and must not count
+    n_head, n_kv, hd, bs, n = 8, 2, 128, 16, len(ctx)
+    mb = -(-max(ctx) // bs)
+    q, kc, ks, vc, vs, tables, cl = paged_case(n, n_head, n_kv, hd, bs, ctx, mb, 98)
+    announce("paged records of an earlier call", ctx)
+    bad = np.where(np.arange(vs.size) % 2, np.nan, np.inf).astype(np.float32)
+    run_paged(q, kc, ks, vc, bad, tables, np.full(n, max(ctx), np.int32), n, n_head, n_kv, hd, bs, mb)
+    got, _ = run_paged(q, kc, ks, vc, vs, tables, cl, n, n_head, n_kv, hd, bs, mb)
+    ref = o.paged_attention_int8(q, kc, ks, vc, vs, tables, cl, n, n_head, n_kv, hd, bs, mb, threads=8)
+    assert_close(got, ref, "paged records of an earlier call")
+
+
 @pytest.mark.parametrize("n_head,n_kv,hd", [(4, 4, 128), (32, 8, 128), (10, 2, 128), (16, 1, 64), (3, 3, 256), (8, 2, 256)])
 @pytest.mark.parametrize("lo,hi", [(0, 1), (0, 127), (0, 128), (0, 129), (5, 20), (17, 1500), (700, 700)])
 def test_flash_tiles(n_head, n_kv, hd, lo, hi):
