@@ -720,16 +720,19 @@ int gemm_mt(size_t M) {
 // Waves of a workgroup, each all 16 MT rows x 32 columns.  Eight (256 columns)
 // share each X tile, one workgroup per CU; up to 64 rows leave registers for
 // two or three workgroups of four per CU, whose stage waits overlap (one layer's
-// seven matrices, 48 rows: 114 us with eight waves, 107 with four; 77 rows with
-// four spill: 145 against 143).
+// seven matrices, 48 rows: 114 us with eight waves, 107 with four).  From 65 rows
+// on four waves spill under the register bound of three workgroups (77 rows: 145
+// us, 143 with eight waves); under a bound for two, 65 to 96 rows do not, and 65
+// measured 123 against 141, which is not used yet.
 constexpr int kNarrowMT = 4;
 constexpr int gemm_waves(int mt) { return mt <= kNarrowMT ? 4 : 8; }
 
 // K splits for a GEMM: none while the tiles fill at least half of the
 // workgroup slots (one per CU, two for up to 48 rows: 17-48 rows 1-5% faster, 64
-// rows 5% slower), since a split costs a partial product
-// per split written and summed again; below that, as many as still fit one
-// round of slots (at most 8, at most one per 256-element block).
+// rows 5% slower; so 49-64 rows have fewer splits than 128-row tiles gave them,
+// and sum in another order), since a split costs a partial product per split
+// written and summed again; below that, as many as still fit one round of slots
+// (at most 8, at most one per 256-element block).
 int gemm_split(size_t M, size_t N, size_t K) {
   const int mt = gemm_mt(M);
   const size_t bm = 16 * (size_t)mt, bn = 32 * (size_t)gemm_waves(mt);

@@ -710,8 +710,8 @@ hipError_t run_ext_as(const uint8_t* w, const float* x, float* y, int out_dim, i
   // more waves, as long as the rows still give every CU its workgroups, and the
   // grid is one workgroup per place, so that x is staged once: IQ4_XS 4096 x
   // 28672 49 -> 24 us, 14336 x 28672 157 -> 67; 14336 x 14336 IQ4_NL 52 -> 41,
-  // IQ3_S 65 -> 55, BF16 77 -> 70; eight rows of 14336 x 4096 IQ4_XS 164 -> 113,
-  // F16 177 -> 112, IQ2_XXS 148 -> 134.
+  // IQ3_S 65 -> 55, BF16 77 -> 70; eight rows of 14336 x 4096 IQ4_XS 164 -> 110,
+  // F16 177 -> 111, IQ2_XXS 146 -> 118.
   const int cus = device_cu_count(), fit = std::max(1, ext_lds_limit() / (int)lds);
   int nw = 4;
   while (nw < kMaxWaves<F, B> && fit * nw < 16 && (out_dim + 2 * nw * R - 1) / (2 * nw * R) >= fit * cus) nw *= 2;

@@ -231,8 +231,8 @@ Q8_MFMA = [  # (out_dim, in_dim, batch): Q8_0 batches of 2-8 on the matrix cores
 @pytest.mark.parametrize("out_dim,in_dim,batch", Q8_MFMA)
 def test_q8_0_small_batch_matrix_cores(out_dim, in_dim, batch):
     # ragged row groups (out_dim not a multiple of 16), every batch size 2-8,
-    # K = 1024 / 2048 / 4096, and a batch of 12 (one chunk of 8 on the matrix
-    # cores, then 4)
+    # K = 1024 / 2048 / 4096, and a batch of 12 (one pass of the kernel for up to
+    # 32 rows)
     w = synth.quant_weights(Q8_0, out_dim, in_dim, 800 + batch + out_dim)
     x = synth.normal_f32((batch, in_dim), 900 + batch)
     announce("q8_0 small batch", out_dim, in_dim, batch)
