@@ -102,10 +102,11 @@ int ssdq_ctx_device(const ssdq_ctx* ctx);
  * synchronize per growth). Growth is refused while the stream is being
  * captured (SSDQ_ERR_HIP): run the call once on the stream before capture, or
  * reserve. ssdq_matvec_dev with several rows takes at most 32 MiB for its K
- * slices (rows x out_dim x 8 bytes a slice, wider matrices in pieces); with less
- * it runs in chunks of 8 rows, each reading W again, instead of failing. No
- * reference counterpart (the reference allocates Metal buffers per call,
- * gpu.rs:492-535). */
+ * slices (rows x out_dim x 8 bytes a slice, wider matrices in pieces). Where
+ * that cannot be had it runs in chunks of 8 rows, each reading W again; they
+ * need none up to in_dim 4096, and the call fails only where their need cannot
+ * be had either. No reference counterpart (the reference allocates Metal buffers
+ * per call, gpu.rs:492-535). */
 /* Grows the stream's scratch buffer of the current device to at least
  * `bytes` now, so later calls up to that need do not allocate. */
 int ssdq_reserve_workspace(size_t bytes, ssdq_stream_t stream);
